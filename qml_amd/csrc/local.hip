@@ -188,6 +188,14 @@ __device__ __forceinline__ void lk_panel_atoms(LkPanel& P, int nm, int a0, int t
     P.row[t] = P.first[lo] + (c - P.soff[lo]);
 }
 
+// Loader of a tile's rows. In the molecules' own order they follow each other from the first one
+// on; in another they are less than 4 GiB in all (checked by the host).
+typedef PanelLoader<double, LAYOUT_ROW, 4, true> LkRows;
+__device__ __forceinline__ LkRows lk_rows(const LkPanel& P, const LkSide& S) {
+    return LkRows(S.X, S.ld, P.row, S.order ? P.lowest : P.row[0],
+                  !S.order && S.ld > LkRows::MAX_LD);
+}
+
 // Add this wave's molecule-pair sums of one sigma to S.
 // Lane layout shared by both tile kinds: value val(r, c) belongs to tile row rowof(r, lane & 15)
 // and tile column colof(c, lane >> 4); byte e of rpack[r] is the panel molecule of tile row
@@ -275,10 +283,7 @@ __global__ __launch_bounds__(256, 2) void local_kernels_kernel(LkSide A, LkSide 
                 if (KIND == LK_GAUSS_MFMA) {
                     WaveTile<double> tile;
                     wave_tile_zero(tile);
-                    typedef PanelLoader<double, LAYOUT_ROW, 4> Rows;
-                    wg_tile_mma_panels<false>(tile, lds, Rows(B.X, B.ld, PB.row, PB.lowest),
-                                              Rows(A.X, A.ld, PA.row, PA.lowest), feats, false,
-                                              false);
+                    wg_tile_mma_panels<false>(tile, lds, lk_rows(PB, B), lk_rows(PA, A), feats);
                     // Lane value (a, b, e): tile row 64 (w >> 1) + 16 b + (lane & 15),
                     // column 64 (w & 1) + 16 a + (lane >> 4) + 4 e.
                     const int rbase = 64 * (w >> 1), cbase = 64 * (w & 1);

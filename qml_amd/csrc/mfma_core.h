@@ -137,14 +137,6 @@ template <typename T>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_view(const T* p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), 0, 0xffffffffu, 0x00027000);
 }
-__device__ __forceinline__ void buffer_load(double& x, __amdgpu_buffer_rsrc_t b, uint32_t lane_off,
-                                            uint32_t off) {
-    x = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, lane_off, off, 0));
-}
-__device__ __forceinline__ void buffer_load(float& x, __amdgpu_buffer_rsrc_t b, uint32_t lane_off,
-                                            uint32_t off) {
-    x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, lane_off, off, 0));
-}
 __device__ __forceinline__ void buffer_load2(double (&x)[2], __amdgpu_buffer_rsrc_t b,
                                              uint32_t lane_off, uint32_t off) {
     const double2 v = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(b, lane_off, off, 0));
@@ -164,34 +156,51 @@ __device__ __forceinline__ void buffer_load2(float (&x)[2], __amdgpu_buffer_rsrc
 // ROW: lane holds features 2(t%8)+{0,1} of rows 8 Q (t/64) + 8u + (t%64)/8.
 // Pairs are loaded whole (16 bytes at any multiple of 8). Where a panel ends, a lane's pair may
 // not start past the last but one row (COL): the lane whose first row is the last one takes the
-// pair's second value for it (`last_row`), and a panel of a single row starts one row earlier
-// (operands of one row only are loaded value by value).
-template <typename T, int LAYOUT, int Q>
+// pair's second value for it (`last_row`), and a panel of a single row starts one row earlier.
+// Operands of one row only (COL), and of a leading dimension whose offsets within a panel pass 32
+// bits (from 4.2e6 doubles on for 128 rows), are loaded value by value at 64-bit addresses
+// (`by_value`), as the last partial chunk is. LISTED: the panel's rows are listed in LDS (ROW).
+template <typename T, int LAYOUT, int Q, bool LISTED = false>
 struct PanelLoader {
     typedef WgShape<Q> S;
     static constexpr int L = 16 * Q;   // lanes per feature (COL)
     static constexpr int PW = 64 / L;  // features per wave and load (COL)
     static constexpr int US = 16 / Q;  // features per workgroup and load (COL)
+    // the largest leading dimension for 32-bit offsets: 16 features (COL) or a panel's rows and 16
+    // features (ROW) span less than 4 GiB
+    static constexpr int64_t MAX_LD = ((int64_t)0xffffffff / (int64_t)sizeof(T) - WgShape<4>::ROWS) /
+                                      (LAYOUT == LAYOUT_COL ? WG_KC : S::ROWS - 1);
     const T* base;    // chunk 0; COL: the wave's first feature, row 0; ROW: its first feature
     int64_t step;     // elements between features (COL)
     uint32_t off[Q];  // COL: [0] the lane's rows; ROW: per u the lane's row and features
     bool last_row;    // COL: the pair's second value is the lane's first row
+    bool by_value;
+    const T* p;       // feature 0 of the panel's first row; LISTED: of row 0
+    int64_t ld;
+    int last;         // last row of the panel
+    const int* idx;   // LISTED: its rows
 
     __device__ __forceinline__ PanelLoader(const Operand<T, LAYOUT>& op, int64_t row0) {
+        static_assert(!LISTED, "an operand's rows follow each other");
         const int lane = threadIdx.x & 63;
         const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         const int64_t rest = op.rows - 1 - row0;  // rows of the panel: 0 .. last
-        const int last = rest < S::ROWS - 1 ? (int)rest : S::ROWS - 1;
+        last = rest < S::ROWS - 1 ? (int)rest : S::ROWS - 1;
+        ld = op.ld;
+        idx = nullptr;
+        by_value = ld > MAX_LD || (LAYOUT == LAYOUT_COL && op.rows == 1);
         if (LAYOUT == LAYOUT_COL) {
             const int back = last == 0 && op.rows > 1 ? 1 : 0;
             const int pair = last + back > 0 ? last + back - 1 : 0;  // last possible pair start
             const int r = 2 * (lane % L);
+            p = op.p + uniform_i64(row0);
             base = op.p + uniform_i64(wave * PW * op.ld + row0 - back);
             step = op.ld;
             off[0] = (uint32_t)(((r < pair ? r : pair) + (lane / L) * op.ld) * sizeof(T));
             last_row = op.rows > 1 && r + back > pair;
         } else {
-            base = op.p + uniform_i64(row0 * op.ld);
+            p = op.p + uniform_i64(row0 * op.ld);
+            base = p;
             step = 1;
 #pragma unroll
             for (int u = 0; u < Q; ++u) {
@@ -201,18 +210,24 @@ struct PanelLoader {
             last_row = false;
         }
     }
-    // ROW: the rows of p listed in idx[0 .. 32 Q - 1] (LDS), none below `first` (the same in every
-    // lane), all within 4 GiB of it.
-    __device__ __forceinline__ PanelLoader(const T* p, int64_t ld, const int* idx, int first) {
-        static_assert(LAYOUT == LAYOUT_ROW, "rows are listed for row-major operands");
+    // The rows of X listed in rows[0 .. 32 Q - 1] (LDS), none below `first` (the same in every
+    // lane). wide: they are not all within 4 GiB of it.
+    __device__ __forceinline__ PanelLoader(const T* X, int64_t ldx, const int* rows, int first,
+                                           bool wide) {
+        static_assert(LISTED && LAYOUT == LAYOUT_ROW, "rows are listed for row-major operands");
         const int lane = threadIdx.x & 63;
         const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        base = p + uniform_i64(first * ld);
+        p = X;
+        ld = ldx;
+        last = S::ROWS - 1;
+        idx = rows;
+        by_value = wide;
+        base = X + uniform_i64(first * ldx);
         step = 1;
 #pragma unroll
         for (int u = 0; u < Q; ++u) {
             const int row = 8 * Q * wave + 8 * u + (lane >> 3);
-            off[u] = (uint32_t)(((idx[row] - first) * ld + 2 * (lane & 7)) * sizeof(T));
+            off[u] = (uint32_t)(((rows[row] - first) * ldx + 2 * (lane & 7)) * sizeof(T));
         }
         last_row = false;
     }
@@ -228,22 +243,27 @@ struct PanelLoader {
 #pragma unroll
         for (int u = 0; u < Q; ++u) buffer_load2(R.v[u], b, lane_off(u), group_off(u));
     }
-    // Registers <- the first k <= 16 features of chunk c, value by value, zeros after. single:
-    // the operand has one row.
-    __device__ __forceinline__ void load_some(PanelRegs<T, Q>& R, int64_t c, int k,
-                                              bool single) const {
+    // Registers <- the first k <= 16 features of chunk c, value by value, zeros after.
+    __device__ __forceinline__ void load_some(PanelRegs<T, Q>& R, int64_t c, int k) const {
         const int lane = threadIdx.x & 63;
         const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        const __amdgpu_buffer_rsrc_t b = buffer_view(base + c * WG_KC * step);
-        const uint32_t second = LAYOUT == LAYOUT_COL && single ? 0u : (uint32_t)sizeof(T);
 #pragma unroll
         for (int u = 0; u < Q; ++u) {
-            const int k0 = LAYOUT == LAYOUT_COL ? wave * PW + lane / L + US * u : 2 * (lane & 7);
-            const int k1 = LAYOUT == LAYOUT_COL ? k0 : k0 + 1;
             R.v[u][0] = T(0);
             R.v[u][1] = T(0);
-            if (k0 < k) buffer_load(R.v[u][0], b, lane_off(u), group_off(u));
-            if (k1 < k) buffer_load(R.v[u][1], b, lane_off(u) + second, group_off(u));
+            if (LAYOUT == LAYOUT_COL) {
+                const int f = wave * PW + lane / L + US * u, r = 2 * (lane % L);
+                const T* x = p + (c * WG_KC + f) * ld;
+                if (f < k) {
+                    R.v[u][0] = x[r < last ? r : last];
+                    R.v[u][1] = x[r + 1 < last ? r + 1 : last];
+                }
+            } else {
+                const int f = 2 * (lane & 7), row = 8 * Q * wave + 8 * u + (lane >> 3);
+                const T* x = p + (LISTED ? idx[row] : row < last ? row : last) * ld + c * WG_KC + f;
+                if (f < k) R.v[u][0] = x[0];
+                if (f + 1 < k) R.v[u][1] = x[1];
+            }
         }
     }
     // LDS panel <- registers.
@@ -306,20 +326,19 @@ __device__ __forceinline__ void half_mma(WaveTile<T, Q>& t, const HalfFrag<T, Q>
 
 // t += F S^T for the panels of two loaders, 32 Q rows each, restricted to this wave's 16 Q x 16 Q
 // block (t -= ... with SUB: the first operand is negated, which is exact): wave w owns rows
-// 16 Q (w & 1) of the first and 16 Q (w >> 1) of the second. single_f / single_s: the operand has
-// one row (COL). `lds` holds WgShape<Q>::LDS elements. All 256 lanes must call this (it has
-// barriers).
-template <bool SUB, typename T, int LF, int LS, int Q>
+// 16 Q (w & 1) of the first and 16 Q (w >> 1) of the second. `lds` holds WgShape<Q>::LDS
+// elements. All 256 lanes must call this (it has barriers).
+template <bool SUB, typename T, int LF, int LS, int Q, bool GF, bool GS>
 __device__ __forceinline__ void wg_tile_mma_panels(WaveTile<T, Q>& t, T* __restrict__ lds,
-                                                   const PanelLoader<T, LF, Q>& lf,
-                                                   const PanelLoader<T, LS, Q>& ls, int64_t kdim,
-                                                   bool single_f, bool single_s) {
+                                                   const PanelLoader<T, LF, Q, GF>& lf,
+                                                   const PanelLoader<T, LS, Q, GS>& ls,
+                                                   int64_t kdim) {
     if (kdim <= 0) return;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int fr = 16 * Q * (w & 1);
     const int sr = 16 * Q * (w >> 1);
     constexpr int WG_PANEL = WgShape<Q>::PANEL;
-    const int64_t whole = single_f || single_s ? 0 : kdim / WG_KC;
+    const int64_t whole = lf.by_value || ls.by_value ? 0 : kdim / WG_KC;
     PanelRegs<T, Q> pf, ps;
     T* cur = lds;
     T* nxt = lds + 2 * WG_PANEL;
@@ -362,12 +381,12 @@ __device__ __forceinline__ void wg_tile_mma_panels(WaveTile<T, Q>& t, T* __restr
         }
         __syncthreads();
     }
-    // the rest of the features, chunk by chunk (one partial chunk, but for single rows)
+    // the rest of the features, chunk by chunk (one partial chunk, or all of them by value)
 #pragma unroll 1
     for (int64_t k0 = whole * WG_KC; k0 < kdim; k0 += WG_KC) {
         const int k = kdim - k0 < WG_KC ? (int)(kdim - k0) : WG_KC;
-        lf.load_some(pf, k0 / WG_KC, k, single_f);
-        ls.load_some(ps, k0 / WG_KC, k, single_s);
+        lf.load_some(pf, k0 / WG_KC, k);
+        ls.load_some(ps, k0 / WG_KC, k);
         lf.store(cur, pf);
         ls.store(cur + WG_PANEL, ps);
         __syncthreads();
@@ -390,7 +409,7 @@ __device__ __forceinline__ void wg_tile_mma_lds(WaveTile<T, Q>& t, T* __restrict
                                                 int64_t kdim) {
     if (kdim <= 0) return;
     wg_tile_mma_panels<SUB>(t, lds, PanelLoader<T, LF, Q>(F, f0), PanelLoader<T, LS, Q>(S, s0),
-                            kdim, LF == LAYOUT_COL && F.rows == 1, LS == LAYOUT_COL && S.rows == 1);
+                            kdim);
 }
 
 // ------------------------------------------------------------------------------------------
