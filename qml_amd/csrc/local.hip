@@ -56,7 +56,7 @@ struct LkSide {
     const int64_t* panels;   // (npanels + 1) first place of each panel in the order
     const int64_t* order;    // (nmol) molecule at each place; null: its index
     const int32_t* count;    // (npanels) leading features that hold every nonzero; null: all
-    int64_t atoms;           // total atoms (rows of X)
+    int64_t atoms;           // total atoms (rows of X): no row beyond them is read
 };
 
 // Set in a panel's feature count: some value of the panel is not finite.
@@ -72,7 +72,8 @@ __device__ __forceinline__ int lk_features(const LkSide& A, const LkSide& B, int
     const int ca = A.count[bi], cb = B.count[bj];
     if (PRODUCT && ((ca | cb) & LK_NOT_FINITE)) return (int)d;
     const int a = ca & ~LK_NOT_FINITE, b = cb & ~LK_NOT_FINITE;
-    return PRODUCT ? (a < b ? a : b) : (a > b ? a : b);
+    const int f = PRODUCT ? (a < b ? a : b) : (a > b ? a : b);
+    return f < d ? f : (int)d;
 }
 
 // count[panel] := 1 + the last feature that is not zero in any of the panel's atom rows, with
@@ -145,15 +146,18 @@ struct LkPanel {
     int row[LK_TILE];        // tile: its row of X (past the last one: the last one's)
 };
 
-// Molecules of panel `p` (nm of them); lanes 0 .. 63 of a wave call it, a barrier follows.
+// Molecules of panel `p` (nm of them), their atoms held to the rows of X; lanes 0 .. 63 of a wave
+// call it, a barrier follows.
 __device__ __forceinline__ void lk_panel_mols(LkPanel& P, const LkSide& S, int p, int nm) {
     const int m = threadIdx.x & 63;
     int n = 0, low = 0x7fffffff;
     if (m < nm) {
         const int64_t at = S.panels[p] + m;
         const int64_t mol = S.order ? S.order[at] : at;
-        const int64_t a0 = S.offsets[mol];
-        n = (int)(S.offsets[mol + 1] - a0);
+        int64_t a0 = S.offsets[mol], a1 = S.offsets[mol + 1];
+        a0 = a0 < 0 ? 0 : a0;
+        a1 = a1 < S.atoms ? a1 : S.atoms;
+        n = a1 > a0 ? (int)(a1 - a0) : 0;
         P.mol[m] = (int)mol;
         P.first[m] = (int)a0;
         low = (int)a0;
@@ -193,6 +197,7 @@ __device__ __forceinline__ void lk_panel_atoms(LkPanel& P, int nm, int a0, int t
 typedef PanelLoader<double, LAYOUT_ROW, 4, true> LkRows;
 __device__ __forceinline__ LkRows lk_rows(const LkPanel& P, const LkSide& S) {
     return LkRows(S.X, S.ld, P.row, S.order ? P.lowest : P.row[0],
+                  S.order ? (int)S.atoms - 1 : P.row[LK_TILE - 1],
                   !S.order && S.ld > LkRows::MAX_LD);
 }
 

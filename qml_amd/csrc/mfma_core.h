@@ -120,8 +120,9 @@ struct PanelRegs {
     T v[Q][2];  // 32 Q x 16 panel / 256 lanes
 };
 
-// Raw buffer view of the memory from p on (4 GiB): loads take a uniform base, a uniform offset
-// and the lane's 32-bit offset, so an address costs no vector registers beyond that offset.
+// Raw buffer view of `bytes` of memory from p on: loads take a uniform base, a uniform offset and
+// the lane's 32-bit offset, so an address costs no vector registers beyond that offset. A load
+// past the view gives zeros.
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -134,8 +135,8 @@ __device__ __forceinline__ int64_t uniform_i64(int64_t v) {
 }
 
 template <typename T>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_view(const T* p) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), 0, 0xffffffffu, 0x00027000);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_view(const T* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), 0, (int)bytes, 0x00027000);
 }
 __device__ __forceinline__ void buffer_load2(double (&x)[2], __amdgpu_buffer_rsrc_t b,
                                              uint32_t lane_off, uint32_t off) {
@@ -173,6 +174,7 @@ struct PanelLoader {
     const T* base;    // chunk 0; COL: the wave's first feature, row 0; ROW: its first feature
     int64_t step;     // elements between features (COL)
     uint32_t off[Q];  // COL: [0] the lane's rows; ROW: per u the lane's row and features
+    uint32_t bytes;   // from a chunk's base to the end of its last feature of the panel's last row
     bool last_row;    // COL: the pair's second value is the lane's first row
     bool by_value;
     const T* p;       // feature 0 of the panel's first row; LISTED: of row 0
@@ -196,12 +198,14 @@ struct PanelLoader {
             p = op.p + uniform_i64(row0);
             base = op.p + uniform_i64(wave * PW * op.ld + row0 - back);
             step = op.ld;
+            bytes = (uint32_t)(((WG_KC - 1 - wave * PW) * op.ld + last + 1 + back) * sizeof(T));
             off[0] = (uint32_t)(((r < pair ? r : pair) + (lane / L) * op.ld) * sizeof(T));
             last_row = op.rows > 1 && r + back > pair;
         } else {
             p = op.p + uniform_i64(row0 * op.ld);
             base = p;
             step = 1;
+            bytes = (uint32_t)((last * op.ld + WG_KC) * sizeof(T));
 #pragma unroll
             for (int u = 0; u < Q; ++u) {
                 const int row = 8 * Q * wave + 8 * u + (lane >> 3);
@@ -210,10 +214,10 @@ struct PanelLoader {
             last_row = false;
         }
     }
-    // The rows of X listed in rows[0 .. 32 Q - 1] (LDS), none below `first` (the same in every
-    // lane). wide: they are not all within 4 GiB of it.
+    // The rows of X listed in rows[0 .. 32 Q - 1] (LDS), from `first` to `highest` (the same in every
+    // lane). wide: they span 4 GiB or more.
     __device__ __forceinline__ PanelLoader(const T* X, int64_t ldx, const int* rows, int first,
-                                           bool wide) {
+                                           int highest, bool wide) {
         static_assert(LISTED && LAYOUT == LAYOUT_ROW, "rows are listed for row-major operands");
         const int lane = threadIdx.x & 63;
         const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -224,6 +228,7 @@ struct PanelLoader {
         by_value = wide;
         base = X + uniform_i64(first * ldx);
         step = 1;
+        bytes = (uint32_t)uniform_i64(((highest - first) * ldx + WG_KC) * (int64_t)sizeof(T));
 #pragma unroll
         for (int u = 0; u < Q; ++u) {
             const int row = 8 * Q * wave + 8 * u + (lane >> 3);
@@ -239,7 +244,7 @@ struct PanelLoader {
     }
     // Registers <- whole chunk c.
     __device__ __forceinline__ void load(PanelRegs<T, Q>& R, int64_t c) const {
-        const __amdgpu_buffer_rsrc_t b = buffer_view(base + c * WG_KC * step);
+        const __amdgpu_buffer_rsrc_t b = buffer_view(base + c * WG_KC * step, bytes);
 #pragma unroll
         for (int u = 0; u < Q; ++u) buffer_load2(R.v[u], b, lane_off(u), group_off(u));
     }

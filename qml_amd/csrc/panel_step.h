@@ -194,8 +194,8 @@ template <typename T>
 __device__ __forceinline__ void step_tile_body(const PanelStep<T>& st, double* __restrict__ lds,
                                                int64_t tile) {
     const int64_t bi = tile % st.strips, bj = tile / st.strips;
-    if (bi <= bj) return;  // on the diagonal or above it
     const int64_t lda = st.lda, m = st.m, ncols = st.ncols;
+    if (bi <= bj || bj * STEP_T >= ncols) return;  // on the diagonal or above it, or none of the step's
     const T* P = st.A + st.w - (int64_t)st.prev * lda;
     T* C = st.A + st.w + st.w * lda;
     Operand<T, LAYOUT_COL> rows{P, lda, m, st.prev};
