@@ -95,6 +95,15 @@ int qmlh_atomic_cm_small(const double *Z, const double *R, const int64_t *offset
                          double central_decay, double interaction_cutoff,
                          double interaction_decay, double *out, int64_t ldo, int32_t *status,
                          int32_t max_atoms, qmlh_stream_t stream);
+/* The rows that qmlh_atomic_cm_small of the same arguments left because their molecules have more
+ * than max_atoms atoms, computed as qmlh_atomic_cm_batch does. first: the device status of that
+ * call; its bits 1 and 4 are added to status. Returns at once on the device if nothing is left. */
+int qmlh_atomic_cm_rest(const double *Z, const double *R, const int64_t *offsets, int64_t nmol,
+                        const int64_t *central, const int64_t *cmol, int64_t nrows,
+                        int32_t size, int32_t sorting, double central_cutoff,
+                        double central_decay, double interaction_cutoff,
+                        double interaction_decay, double *out, int64_t ldo, int32_t *status,
+                        const int32_t *first, int32_t max_atoms, qmlh_stream_t stream);
 /* Rows of molecules with more than QMLH_ACM_MAX_ATOMS atoms (up to max_atoms), which
  * qmlh_atomic_cm_batch reports with status bit 2 and leaves zero: the same rows, with each
  * molecule staged in a slice of the workspace instead of LDS. Same arguments and status bits

@@ -59,6 +59,8 @@ _SIGNATURES = {
                                             _f64, _f64, _f64, _f64, _vp, _i64, _vp, _vp]),
     "qmlh_atomic_cm_small": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _f64,
                                             _f64, _f64, _f64, _vp, _i64, _vp, _i32, _vp]),
+    "qmlh_atomic_cm_rest": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _f64,
+                                           _f64, _f64, _f64, _vp, _i64, _vp, _vp, _i32, _vp]),
     "qmlh_atomic_cm_large_workspace": (_sz, [_i64, _i32]),
     "qmlh_atomic_cm_large": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32,
                                             _f64, _f64, _f64, _f64, _vp, _i64, _vp, _i64, _vp,

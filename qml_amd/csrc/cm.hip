@@ -463,12 +463,16 @@ __device__ __forceinline__ double acm_pair(const double* sR, const double* sZ, i
 // status bits: 1 a central atom needs more than `size` rows; 2 a molecule has more than
 // QMLH_ACM_MAX_ATOMS atoms; 4 a central atom or molecule index is out of range. The row of
 // such a case is written as zeros.
+// first (null: all rows are computed): the status of atomic_cm_small_kernel over the same rows. Its
+// bits 1 and 4 are taken over, and where it has bit 2, the rows of molecules of more than
+// first_atoms atoms, which that kernel left, are computed here and the others kept.
 template <bool ROWNORM>
 __global__ __launch_bounds__(CM_WAVE) void atomic_cm_kernel(
     const double* __restrict__ Z, const double* __restrict__ R,
     const int64_t* __restrict__ offsets, int64_t nmol, const int64_t* __restrict__ central,
     const int64_t* __restrict__ cmol, int64_t nrows, int size, AcmParams p, int64_t ldo,
-    double* __restrict__ out, int32_t* __restrict__ status) {
+    double* __restrict__ out, int32_t* __restrict__ status,
+    const int32_t* __restrict__ first, int first_atoms) {
     __shared__ double sR[3 * ACM_MAX_ATOMS];
     __shared__ double sZ[ACM_MAX_ATOMS];
     __shared__ double sDk[ACM_MAX_ATOMS];
@@ -477,9 +481,19 @@ __global__ __launch_bounds__(CM_WAVE) void atomic_cm_kernel(
     const int lane = threadIdx.x;
     const int d = size * (size + 1) / 2;
 
+    if (first) {
+        const int32_t before = *first;
+        if (blockIdx.x == 0 && lane == 0 && status && (before & ~2)) atomicOr(status, before & ~2);
+        if (!(before & 2)) return;
+    }
     for (int64_t row = blockIdx.x; row < nrows; row += gridDim.x) {
         double* dst = out + row * ldo;
         const int64_t mol = cmol[row];
+        if (first) {
+            if (mol < 0 || mol >= nmol) continue;
+            const int64_t n = offsets[mol + 1] - offsets[mol];
+            if (n >= 0 && n <= first_atoms) continue;
+        }
         int bad = 0;
         int64_t a0 = 0, n64 = 0, k64 = central[row];
         if (mol < 0 || mol >= nmol) {
@@ -960,6 +974,37 @@ static AcmParams acm_params(double cc, double cd, double ic, double id) {
 
 }  // namespace qmlh
 
+namespace qmlh {
+
+static int atomic_cm_rows(const char* who, const double* Z, const double* R,
+                          const int64_t* offsets, int64_t nmol, const int64_t* central,
+                          const int64_t* cmol, int64_t nrows, int32_t size, int32_t sorting,
+                          const AcmParams& p, double* out, int64_t ldo, int32_t* status,
+                          const int32_t* first, int32_t first_atoms, int64_t grid, hipStream_t s) {
+    if (nrows < 0 || nmol < 0) return set_error(QMLH_ERR_ARG, "%s: negative count", who);
+    if (size < 1 || size > QMLH_CM_MAX_SIZE)
+        return set_error(QMLH_ERR_ARG, "%s: size %d outside [1, %d]", who, size,
+                         QMLH_CM_MAX_SIZE);
+    if (sorting != QMLH_ACM_ROW_NORM && sorting != QMLH_ACM_DISTANCE)
+        return set_error(QMLH_ERR_ARG, "%s: unknown sorting %d", who, sorting);
+    int64_t d = (int64_t)size * (size + 1) / 2;
+    if (ldo < d) return set_error(QMLH_ERR_ARG, "%s: ldo %lld < %lld", who, (long long)ldo,
+                                  (long long)d);
+    if (nrows == 0) return QMLH_OK;
+    if (!Z || !R || !offsets || !central || !cmol || !out)
+        return set_error(QMLH_ERR_ARG, "%s: null pointer", who);
+    TimerScope ts(QMLH_TIMER_CM, (double)nrows, s);
+    hipLaunchKernelGGL((sorting == QMLH_ACM_ROW_NORM ? atomic_cm_kernel<true>
+                                                     : atomic_cm_kernel<false>),
+                       dim3((unsigned)(nrows < grid ? nrows : grid)), dim3(CM_WAVE), 0, s, Z, R,
+                       offsets, nmol, central, cmol, nrows, (int)size, p, ldo, out, status, first,
+                       (int)first_atoms);
+    QMLH_CHECK_LAUNCH(who);
+    return QMLH_OK;
+}
+
+}  // namespace qmlh
+
 extern "C" int qmlh_atomic_cm_batch(const double* Z, const double* R, const int64_t* offsets,
                                     int64_t nmol, const int64_t* central, const int64_t* cmol,
                                     int64_t nrows, int32_t size, int32_t sorting,
@@ -968,32 +1013,28 @@ extern "C" int qmlh_atomic_cm_batch(const double* Z, const double* R, const int6
                                     double* out, int64_t ldo, int32_t* status,
                                     qmlh_stream_t stream) {
     using namespace qmlh;
-    if (nrows < 0 || nmol < 0) return set_error(QMLH_ERR_ARG, "atomic_cm_batch: negative count");
-    if (size < 1 || size > QMLH_CM_MAX_SIZE)
-        return set_error(QMLH_ERR_ARG, "atomic_cm_batch: size %d outside [1, %d]", size,
-                         QMLH_CM_MAX_SIZE);
-    if (sorting != QMLH_ACM_ROW_NORM && sorting != QMLH_ACM_DISTANCE)
-        return set_error(QMLH_ERR_ARG, "atomic_cm_batch: unknown sorting %d", sorting);
-    int64_t d = (int64_t)size * (size + 1) / 2;
-    if (ldo < d) return set_error(QMLH_ERR_ARG, "atomic_cm_batch: ldo %lld < %lld",
-                                  (long long)ldo, (long long)d);
-    if (nrows == 0) return QMLH_OK;
-    if (!Z || !R || !offsets || !central || !cmol || !out)
-        return set_error(QMLH_ERR_ARG, "atomic_cm_batch: null pointer");
-    const AcmParams p = acm_params(central_cutoff, central_decay, interaction_cutoff,
-                                   interaction_decay);
-    int64_t grid = nrows < 262144 ? nrows : 262144;
-    hipStream_t s = (hipStream_t)stream;
-    TimerScope ts(QMLH_TIMER_CM, (double)nrows, s);
-    if (sorting == QMLH_ACM_ROW_NORM)
-        hipLaunchKernelGGL(atomic_cm_kernel<true>, dim3((unsigned)grid), dim3(CM_WAVE), 0, s, Z,
-                           R, offsets, nmol, central, cmol, nrows, (int)size, p, ldo, out, status);
-    else
-        hipLaunchKernelGGL(atomic_cm_kernel<false>, dim3((unsigned)grid), dim3(CM_WAVE), 0, s,
-                           Z, R, offsets, nmol, central, cmol, nrows, (int)size, p, ldo, out,
-                           status);
-    QMLH_CHECK_LAUNCH("atomic_cm_batch launch");
-    return QMLH_OK;
+    return atomic_cm_rows("atomic_cm_batch", Z, R, offsets, nmol, central, cmol, nrows, size,
+                          sorting,
+                          acm_params(central_cutoff, central_decay, interaction_cutoff,
+                                     interaction_decay),
+                          out, ldo, status, nullptr, 0, 262144, (hipStream_t)stream);
+}
+
+extern "C" int qmlh_atomic_cm_rest(const double* Z, const double* R, const int64_t* offsets,
+                                   int64_t nmol, const int64_t* central, const int64_t* cmol,
+                                   int64_t nrows, int32_t size, int32_t sorting,
+                                   double central_cutoff, double central_decay,
+                                   double interaction_cutoff, double interaction_decay,
+                                   double* out, int64_t ldo, int32_t* status,
+                                   const int32_t* first, int32_t max_atoms, qmlh_stream_t stream) {
+    using namespace qmlh;
+    if (!first) return set_error(QMLH_ERR_ARG, "atomic_cm_rest: null pointer");
+    // few workgroups: where no row is left, the launch is all that the call takes
+    return atomic_cm_rows("atomic_cm_rest", Z, R, offsets, nmol, central, cmol, nrows, size,
+                          sorting,
+                          acm_params(central_cutoff, central_decay, interaction_cutoff,
+                                     interaction_decay),
+                          out, ldo, status, first, max_atoms, 4096, (hipStream_t)stream);
 }
 
 extern "C" int qmlh_atomic_cm_small(const double* Z, const double* R, const int64_t* offsets,

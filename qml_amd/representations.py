@@ -100,8 +100,10 @@ def generate_atomic_coulomb_matrices_device(Zd, Rd, Od, central, cmol, size: int
     (nmol+1,), central i64 (rows,) central atom within its molecule, cmol i64 (rows,) its
     molecule. Returns ``(out, status)``: the (rows, ld) FP64 device tensor (pad columns zero)
     and the device status word (bit 1: a central atom needs more than ``size`` rows; bit 4: an
-    index out of range). max_atoms: the largest molecule (read from ``offsets`` when None);
-    molecules above 256 atoms go through the global-memory kernel (qmlh_atomic_cm_large)."""
+    index out of range; bit 2: a molecule has more than 256 atoms and ``max_atoms`` does not say
+    so; such rows are zero). max_atoms: the largest molecule (read from ``offsets`` when None);
+    up to 256 it only chooses the kernel, molecules above 256 atoms go through the global-memory
+    kernel (qmlh_atomic_cm_large)."""
     import torch
 
     if sorting not in _ACM_SORTINGS:
@@ -118,11 +120,17 @@ def generate_atomic_coulomb_matrices_device(Zd, Rd, Od, central, cmol, size: int
             _lib.ptr(cmol), rows, size, _ACM_SORTINGS[sorting], float(central_cutoff),
             float(central_decay), float(interaction_cutoff), float(interaction_decay),
             _lib.ptr(out), ld)
+    hinted = max_atoms is not None
     if max_atoms is None:
         max_atoms = int((Od[1:] - Od[:-1]).max()) if Od.shape[0] > 1 else 0
     if max_atoms <= _lib.ACM_SMALL_ATOMS:
-        _lib.check(L.qmlh_atomic_cm_small(*args, _lib.ptr(status), max_atoms,
+        small = max(0, int(max_atoms))
+        first = torch.zeros(1, dtype=torch.int32, device=Od.device) if hinted else status
+        _lib.check(L.qmlh_atomic_cm_small(*args, _lib.ptr(first), small,
                                           _lib.stream_handle(stream)))
+        if hinted:  # a molecule may still be larger than the caller says
+            _lib.check(L.qmlh_atomic_cm_rest(*args, _lib.ptr(status), _lib.ptr(first), small,
+                                             _lib.stream_handle(stream)))
         return out, status
     if max_atoms <= _lib.ACM_MAX_ATOMS:
         _lib.check(L.qmlh_atomic_cm_batch(*args, _lib.ptr(status), _lib.stream_handle(stream)))
