@@ -99,9 +99,9 @@ def cho_solve(A, y):
     info = potrf_device(Ad, n)
     xd = torch.from_numpy(np.array(y, dtype=np.float64)).to(device())
     potrs_device(Ad, n, xd)
-    _copy_lower_to_upper(A)  # while the device works on its copy
     x[:] = xd.cpu().numpy()
     print_potrf_warning(int(info.item()))
+    _copy_lower_to_upper(A)  # last: A is the caller's until the device's work has ended
     return x
 
 
