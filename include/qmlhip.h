@@ -493,6 +493,7 @@ int qmlh_local_kernels(int32_t kind, const double *A, int64_t atomsA, int64_t ld
  * molecule cost most of that padding only where molecules of unlike size share a panel, so an
  * order by size makes the call faster. With norms (expanded form), an ordered side's
  * representations take less than 4 GiB. QMLH_SYMMETRIC: orderA == orderB as well. */
+#define QMLH_LOCAL_COUNT_PAIRS 512 /* calls of no more panel pairs skip nothing */
 size_t qmlh_local_kernels_workspace(int64_t npA, int64_t npB);
 int qmlh_local_kernels_ordered(int32_t kind, const double *A, int64_t atomsA, int64_t lda,
                                const double *normsA, const int64_t *offsA, const int64_t *panelsA,

@@ -23,6 +23,7 @@ LOWER = 2
 CM_MAX_SIZE = 256
 ACM_MAX_ATOMS = 256
 ACM_SMALL_ATOMS = 32
+LOCAL_COUNT_PAIRS = 512
 ACM_ROW_NORM, ACM_DISTANCE = 0, 1
 
 _lock = threading.Lock()

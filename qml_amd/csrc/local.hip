@@ -44,7 +44,7 @@ static_assert(LK_MOLS == 16, "one 16-wide MFMA block of molecules per panel side
 // Workgroups per launch; larger panel-pair counts are covered by a grid-stride loop.
 static constexpr int64_t LK_MAX_GRID = 1 << 20;
 static constexpr int LK_COUNT_LANES = 1024;
-static constexpr int64_t LK_COUNT_PAIRS = 512;
+static constexpr int64_t LK_COUNT_PAIRS = QMLH_LOCAL_COUNT_PAIRS;
 
 enum { LK_GAUSS_MFMA = 0, LK_GAUSS_VALU = 1, LK_LAPLACE = 2 };
 

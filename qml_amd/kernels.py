@@ -241,8 +241,8 @@ class LocalSet:
     launch needs: rows (atoms, ld) FP64, atom offsets on the device, the molecules ordered by
     size (largest first, so that the panels of a launch hold molecules of like size and skip the
     padding of the small ones; None for 4 GiB of rows and more, which the expanded form takes in
-    their own order only) with the panels of that order, and (for the Gaussian expanded form)
-    the squared row norms."""
+    their own order only) with the panels of that order and of the molecules' own, and (for the
+    Gaussian expanded form) the squared row norms."""
 
     def __init__(self, X, n_atoms, ld: int | None = None):
         import torch
@@ -259,17 +259,18 @@ class LocalSet:
             Xh = np.asarray(X, dtype=np.float64).reshape(self.atoms, -1)
             self.d = Xh.shape[1]
             self.X = rows_to_device(Xh, ld)
-        dev = self.X.device
-        self.order_d = None
-        ordered = self.offsets
+        order, ordered = np.zeros(0, dtype=np.int64), self.offsets
         if self.X.numel() < 1 << 29:
             order = np.argsort(-counts, kind="stable")
-            self.order_d = torch.from_numpy(order).to(dev)
             ordered = np.zeros_like(self.offsets)
             np.cumsum(counts[order], out=ordered[1:])
-        self.panels = local_panels(ordered)
-        self.offsets_d = torch.from_numpy(self.offsets).to(dev)
-        self.panels_d = torch.from_numpy(self.panels).to(dev)
+        self.panels, self.own_panels = local_panels(ordered), local_panels(self.offsets)
+        parts = (self.offsets, self.panels, self.own_panels, order)
+        ends = np.cumsum([p.size for p in parts])
+        buf = torch.from_numpy(np.concatenate(parts)).to(self.X.device)
+        self.offsets_d, self.panels_d, self.own_panels_d, order_d = (
+            buf[e - p.size:e] for p, e in zip(parts, ends))
+        self.order_d = order_d if order.size else None
         self._norms = None
         self._maxnorm = None
 
@@ -287,6 +288,21 @@ class LocalSet:
         if self._maxnorm is None:
             self._maxnorm = float(self.norms().max().item()) if self.atoms else 0.0
         return self._maxnorm
+
+
+def _local_orders(SA: LocalSet, SB: LocalSet, symmetric: bool):
+    """(order, panels) of both sides for a call. Up to LOCAL_COUNT_PAIRS panel pairs no padding is
+    skipped, and an order by size only makes more panels (16 small molecules do not fill one), so
+    such a call takes the molecules' own order where that has no more panel pairs: 192 molecules of
+    5 to 23 atoms are 253 pairs and not 276, one round of the 256 CUs and not two."""
+    def pairs(a, b):
+        return a * (a + 1) // 2 if symmetric else a * b
+
+    ordered = pairs(SA.panels.size - 1, SB.panels.size - 1)
+    if ordered <= _lib.LOCAL_COUNT_PAIRS and \
+            pairs(SA.own_panels.size - 1, SB.own_panels.size - 1) <= ordered:
+        return [(None, S.own_panels_d) for S in (SA, SB)]
+    return [(S.order_d, S.panels_d) for S in (SA, SB)]
 
 
 def local_kernels_device(kind: int, SA: LocalSet, SB: LocalSet, sigmas, symmetric=False,
@@ -313,14 +329,16 @@ def local_kernels_device(kind: int, SA: LocalSet, SB: LocalSet, sigmas, symmetri
         if expanded:
             nA, nB = SA.norms(), SB.norms()
     L = _lib.lib()
-    ws_bytes = L.qmlh_local_kernels_workspace(SA.npanels, SB.npanels)
+    (oA, pA), (oB, pB) = _local_orders(SA, SB, symmetric)
+    npA, npB = pA.numel() - 1, pB.numel() - 1
+    ws_bytes = L.qmlh_local_kernels_workspace(npA, npB)
     with torch.cuda.stream(stream) if stream is not None else contextlib.nullcontext():
         ws = torch.empty(max(1, (ws_bytes + 7) // 8), dtype=torch.float64, device=SA.X.device)
     _lib.check(L.qmlh_local_kernels_ordered(
         kind, _lib.ptr(SA.X), SA.atoms, SA.X.shape[1], _lib.ptr(nA) if nA is not None else None,
-        _lib.ptr(SA.offsets_d), _lib.ptr(SA.panels_d), _lib.ptr(SA.order_d), SA.npanels,
+        _lib.ptr(SA.offsets_d), _lib.ptr(pA), _lib.ptr(oA), npA,
         _lib.ptr(SB.X), SB.atoms, SB.X.shape[1], _lib.ptr(nB) if nB is not None else None,
-        _lib.ptr(SB.offsets_d), _lib.ptr(SB.panels_d), _lib.ptr(SB.order_d), SB.npanels, SA.d,
+        _lib.ptr(SB.offsets_d), _lib.ptr(pB), _lib.ptr(oB), npB, SA.d,
         sig.ctypes.data, sig.size, _lib.ptr(K), SA.nmol, SA.nmol * SB.nmol,
         _lib.SYMMETRIC if symmetric else 0, _lib.ptr(ws), ws.numel() * 8,
         _lib.stream_handle(stream)))
