@@ -34,6 +34,10 @@ inline int check_hip(hipError_t e, const char* what) {
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline int64_t round_up(int64_t a, int64_t b) { return ceil_div(a, b) * b; }
 
+// Workgroups of 256 lanes that a launch of work in a grid-stride loop takes at most: a grid of 2^32
+// lanes and more is cut short without an error.
+static constexpr int64_t MAX_GRID = (int64_t)1 << 23;
+
 // FP64 MFMA operand/accumulator vector types.
 typedef double double4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));

@@ -45,16 +45,16 @@ static int64_t kernel_tiles(int64_t na, int64_t nb, bool sym, int64_t side) {
 __global__ __launch_bounds__(256) void row_sqnorms_kernel(const double* __restrict__ X,
                                                           int64_t n, int64_t ld, int64_t d,
                                                           double* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= n) return;
     const int lane = threadIdx.x & 63;
-    const double* x = X + i * ld;
-    double s = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); i < n; i += (int64_t)gridDim.x * 4) {
+        const double* x = X + i * ld;
+        double s = 0.0;
 #pragma unroll 8
-    for (int64_t k = lane; k < d; k += 64) s = fma(x[k], x[k], s);
+        for (int64_t k = lane; k < d; k += 64) s = fma(x[k], x[k], s);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s = s + __shfl_xor(s, off, 64);
-    if (lane == 0) out[i] = s;
+        for (int off = 32; off > 0; off >>= 1) s = s + __shfl_xor(s, off, 64);
+        if (lane == 0) out[i] = s;
+    }
 }
 
 __global__ void exp_scale_kernel(const double* __restrict__ norms, int64_t n, double scale,
@@ -259,8 +259,8 @@ extern "C" int qmlh_row_sqnorms(const double* X, int64_t n, int64_t ldx, int64_t
     if (n < 0 || d < 0 || ldx < d) return set_error(QMLH_ERR_ARG, "row_sqnorms: bad shape");
     if (n == 0) return QMLH_OK;
     if (!X || !norms) return set_error(QMLH_ERR_ARG, "row_sqnorms: null pointer");
-    if (ceil_div(n, 4) > 0x7fffffffLL) return set_error(QMLH_ERR_ARG, "row_sqnorms: grid too large");
-    hipLaunchKernelGGL(row_sqnorms_kernel, dim3((unsigned)ceil_div(n, 4)), dim3(256), 0,
+    const int64_t grid = ceil_div(n, 4) < MAX_GRID ? ceil_div(n, 4) : MAX_GRID;
+    hipLaunchKernelGGL(row_sqnorms_kernel, dim3((unsigned)grid), dim3(256), 0,
                        (hipStream_t)stream, X, n, ldx, d, norms);
     QMLH_CHECK_LAUNCH("row_sqnorms launch");
     return QMLH_OK;

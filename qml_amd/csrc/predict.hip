@@ -219,17 +219,20 @@ __global__ __launch_bounds__(256) void predict_reduce_kernel(const double* __res
                                                              double* __restrict__ y) {
     __shared__ double red[16][17];
     const int qi = threadIdx.x & 15, i = threadIdx.x >> 4;
-    const int64_t q = (int64_t)blockIdx.x * 16 + qi;
-    const double* p = part + (q < m ? q : m - 1);
-    double s = 0.0;
+    for (int64_t q0 = (int64_t)blockIdx.x * 16; q0 < m; q0 += (int64_t)gridDim.x * 16) {
+        const int64_t q = q0 + qi;
+        const double* p = part + (q < m ? q : m - 1);
+        double s = 0.0;
 #pragma unroll 8
-    for (int64_t c = i; c < nchunks; c += 16) s = s + p[c * m];
-    red[i][qi] = s;
-    __syncthreads();
-    if (i == 0 && q < m) {
-        double v = red[0][qi];
-        for (int k = 1; k < 16; ++k) v = v + red[k][qi];
-        y[q] = v;
+        for (int64_t c = i; c < nchunks; c += 16) s = s + p[c * m];
+        red[i][qi] = s;
+        __syncthreads();
+        if (i == 0 && q < m) {
+            double v = red[0][qi];
+            for (int k = 1; k < 16; ++k) v = v + red[k][qi];
+            y[q] = v;
+        }
+        __syncthreads();  // the sums are read before the next queries'
     }
 }
 
@@ -307,8 +310,9 @@ static int predict_impl(int32_t kind, const double* Xq, int64_t m, int64_t ldq,
                            dim3(256), 0, s, Xq, ldq, m, Xt, ldt, n, alpha, d, -1.0 / sigma, part);
     }
     QMLH_CHECK_LAUNCH("krr_predict launch");
-    hipLaunchKernelGGL(predict_reduce_kernel, dim3((unsigned)ceil_div(m, 16)), dim3(256), 0, s,
-                       part, m, nchunks, y);
+    const int64_t sums = ceil_div(m, 16) < MAX_GRID ? ceil_div(m, 16) : MAX_GRID;
+    hipLaunchKernelGGL(predict_reduce_kernel, dim3((unsigned)sums), dim3(256), 0, s, part, m,
+                       nchunks, y);
     QMLH_CHECK_LAUNCH("krr_predict reduce launch");
     return QMLH_OK;
 }
