@@ -107,10 +107,12 @@ __device__ __forceinline__ void bk_pivot(double* __restrict__ A, int64_t n, int6
         }
         double rowmax;
         int64_t jmax;
+        // read before the search's barriers: the first thread may interchange it right after them
+        const double absimax = fabs(at(imax, imax));
         bk_argmax(v, vi, s_v, s_i, rowmax, jmax);
         if (absakk >= alpha * colmax * (colmax / rowmax)) {
             kp = k;
-        } else if (fabs(at(imax, imax)) >= alpha * rowmax) {
+        } else if (absimax >= alpha * rowmax) {
             kp = imax;
         } else {
             kp = imax;
