@@ -46,7 +46,8 @@ static constexpr int64_t LK_MAX_GRID = 1 << 20;
 static constexpr int LK_COUNT_LANES = 1024;
 static constexpr int64_t LK_COUNT_PAIRS = QMLH_LOCAL_COUNT_PAIRS;
 
-enum { LK_GAUSS_MFMA = 0, LK_GAUSS_VALU = 1, LK_LAPLACE = 2 };
+// LK_GAUSS_WIDE: the expanded form for rows whose offsets within a tile pass 32 bits.
+enum { LK_GAUSS_MFMA = 0, LK_GAUSS_VALU = 1, LK_LAPLACE = 2, LK_GAUSS_WIDE = 3 };
 
 struct LkSide {
     const double* X;
@@ -195,10 +196,10 @@ __device__ __forceinline__ void lk_panel_atoms(LkPanel& P, int nm, int a0, int t
 // Loader of a tile's rows. In the molecules' own order they follow each other from the first one
 // on; in another they are less than 4 GiB in all (checked by the host).
 typedef PanelLoader<double, LAYOUT_ROW, 4, true> LkRows;
+template <bool WIDE>
 __device__ __forceinline__ LkRows lk_rows(const LkPanel& P, const LkSide& S) {
     return LkRows(S.X, S.ld, P.row, S.order ? P.lowest : P.row[0],
-                  S.order ? (int)S.atoms - 1 : P.row[LK_TILE - 1],
-                  !S.order && S.ld > LkRows::MAX_LD);
+                  S.order ? (int)S.atoms - 1 : P.row[LK_TILE - 1], WIDE);
 }
 
 // Add this wave's molecule-pair sums of one sigma to S.
@@ -244,8 +245,8 @@ __global__ __launch_bounds__(256, 2) void local_kernels_kernel(LkSide A, LkSide 
                                                                int64_t ldk, int64_t sstride,
                                                                int symmetric, int tiles_a,
                                                                int ntiles) {
-    __shared__ __attribute__((aligned(16))) double lds[KIND == LK_GAUSS_MFMA ? WG_LDS_ELEMS
-                                                                              : PT_ELEMS];
+    constexpr bool WIDE = KIND == LK_GAUSS_WIDE, PRODUCT = KIND == LK_GAUSS_MFMA || WIDE;
+    __shared__ __attribute__((aligned(16))) double lds[PRODUCT ? WG_LDS_ELEMS : PT_ELEMS];
     __shared__ double acc[LK_NS][LK_MOLS * LK_MOLS];
     __shared__ LkPanel PA, PB;
 
@@ -278,17 +279,18 @@ __global__ __launch_bounds__(256, 2) void local_kernels_kernel(LkSide A, LkSide 
         else if (w == 1) lk_panel_mols(PB, B, bj, nmb);
         __syncthreads();
         const int atoms_a = PA.soff[nma], atoms_b = PB.soff[nmb];
-        const int feats = lk_features<KIND == LK_GAUSS_MFMA>(A, B, bi, bj, d);
+        const int feats = lk_features<PRODUCT>(A, B, bi, bj, d);
 
         for (int r0 = 0; r0 < atoms_a; r0 += LK_TILE) {
             for (int c0 = 0; c0 < atoms_b; c0 += LK_TILE) {
                 if (t < LK_TILE) lk_panel_atoms(PA, nma, r0, t);
                 else lk_panel_atoms(PB, nmb, c0, t - LK_TILE);
                 __syncthreads();
-                if (KIND == LK_GAUSS_MFMA) {
+                if (PRODUCT) {
                     WaveTile<double> tile;
                     wave_tile_zero(tile);
-                    wg_tile_mma_panels<false>(tile, lds, lk_rows(PB, B), lk_rows(PA, A), feats);
+                    wg_tile_mma_panels<false>(tile, lds, lk_rows<WIDE>(PB, B), lk_rows<WIDE>(PA, A),
+                                              feats);
                     // Lane value (a, b, e): tile row 64 (w >> 1) + 16 b + (lane & 15),
                     // column 64 (w & 1) + 16 a + (lane >> 4) + 4 e.
                     const int rbase = 64 * (w >> 1), cbase = 64 * (w & 1);
@@ -501,7 +503,9 @@ static int local_kernels(int32_t kind, const double* A, int64_t atomsA, int64_t 
             sg.inv[q] = kind == QMLH_PAIR_GAUSSIAN ? -0.5 / (sig * sig) : -1.0 / sig;
         }
         const int sym = symmetric ? 1 : 0;
-        if (mfma) lk_launch<LK_GAUSS_MFMA>(grid, s, sa, sb, d, sg, K, ldk, sstride, sym, npA);
+        if (mfma && ((!orderA && lda > LkRows::MAX_LD) || (!orderB && ldb > LkRows::MAX_LD)))
+            lk_launch<LK_GAUSS_WIDE>(grid, s, sa, sb, d, sg, K, ldk, sstride, sym, npA);
+        else if (mfma) lk_launch<LK_GAUSS_MFMA>(grid, s, sa, sb, d, sg, K, ldk, sstride, sym, npA);
         else if (kind == QMLH_PAIR_GAUSSIAN)
             lk_launch<LK_GAUSS_VALU>(grid, s, sa, sb, d, sg, K, ldk, sstride, sym, npA);
         else lk_launch<LK_LAPLACE>(grid, s, sa, sb, d, sg, K, ldk, sstride, sym, npA);

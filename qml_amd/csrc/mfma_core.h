@@ -138,6 +138,13 @@ template <typename T>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_view(const T* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), 0, (int)bytes, 0x00027000);
 }
+template <typename T>
+__device__ __forceinline__ T buffer_load(__amdgpu_buffer_rsrc_t b, uint32_t lane_off) {
+    if constexpr (sizeof(T) == 8)
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(b, lane_off, 0, 0));
+    else
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(b, lane_off, 0, 0));
+}
 __device__ __forceinline__ void buffer_load2(double (&x)[2], __amdgpu_buffer_rsrc_t b,
                                              uint32_t lane_off, uint32_t off) {
     const double2 v = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(b, lane_off, off, 0));
@@ -265,6 +272,12 @@ struct PanelLoader {
                 }
             } else {
                 const int f = 2 * (lane & 7), row = 8 * Q * wave + 8 * u + (lane >> 3);
+                if (LISTED && !by_value) {  // nothing kept for it but the offsets
+                    const __amdgpu_buffer_rsrc_t b = buffer_view(base + c * WG_KC, bytes);
+                    if (f < k) R.v[u][0] = buffer_load<T>(b, off[u]);
+                    if (f + 1 < k) R.v[u][1] = buffer_load<T>(b, off[u] + (uint32_t)sizeof(T));
+                    continue;
+                }
                 const T* x = p + (LISTED ? idx[row] : row < last ? row : last) * ld + c * WG_KC + f;
                 if (f < k) R.v[u][0] = x[0];
                 if (f + 1 < k) R.v[u][1] = x[1];
