@@ -554,12 +554,14 @@ __global__ __launch_bounds__(256) void bkb_pivot_kernel(double* __restrict__ A, 
     if (S.need2) {
         double rowmax;
         int64_t jmax;
+        // read before the reduction's barriers: the interchange right after them writes it
+        const double absimax = fabs(W[imax + (int64_t)(j + 1) * ldw]);
         bkb_reduce(part, gridDim.x, rowmax, jmax, s_v, s_i);
         const double alpha = (1.0 + sqrt(17.0)) / 8.0;
         if (S.absakk >= alpha * S.colmax * (S.colmax / rowmax)) {
             kp = k;
             kstep = 1;
-        } else if (fabs(W[imax + (int64_t)(j + 1) * ldw]) >= alpha * rowmax) {
+        } else if (absimax >= alpha * rowmax) {
             kp = imax;
             kstep = 1;
             copy = true;  // W(:, j) := W(:, j + 1)
