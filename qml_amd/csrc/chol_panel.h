@@ -20,8 +20,7 @@ __device__ __forceinline__ double readlane_f64(double v, int lane) {
 
 // Packed lower triangle of a 64 x 64 block in LDS, column-major: element (i, j), i >= j, at
 // pk(i, j); column j holds rows j .. 63. 2080 doubles (16.6 KB) instead of a padded square
-// (33 KB), so the panel kernels fit in the LDS the trailing-update workgroups leave free and run
-// beside them. Wherever the loops are unrolled the index is a compile-time constant (+ lane).
+// (33 KB). Wherever the loops are unrolled the index is a compile-time constant (+ lane).
 static constexpr int CP_PACK = CP_B * (CP_B + 1) / 2;
 __host__ __device__ constexpr int pk(int i, int j) { return j * CP_B - (j * (j - 1)) / 2 + (i - j); }
 
@@ -250,7 +249,7 @@ struct TrsmRows {
     double4_t x[4];
 };
 
-// Diagonal block of a sub-panel, one workgroup: factor the w x w block at A in wave 0, write
+// Diagonal block of a sub-panel, one workgroup: factor the w x w block at A (potf2_block64), write
 // L back, set info = col_base + c + 1 on a failed pivot. `info` already set: nothing is done.
 // sp: CP_PACK doubles of LDS (potf2_body brings its own; a kernel that has LDS to spare at
 // that point passes it).

@@ -181,7 +181,7 @@ __global__ __launch_bounds__(CM_WAVE) void cm_kernel(const double* __restrict__ 
 // marks picked atoms). Otherwise one lane makes the selection step by step.
 // Every value is rounded as above, so the output's bits do not depend on which kernel runs.
 // Bound by instruction issue (IEEE square root and division per pair, index arithmetic per entry):
-// 50,000 molecules of 5-29 atoms, size 29: 364 -> 84 us = 2.4 TB/s of the
+// 50,000 molecules of 5-29 atoms, size 29: 352 -> 84 us = 2.4 TB/s of the
 // rows and atoms (unsorted: 76 -> 52 us = 3.9 TB/s).
 // ------------------------------------------------------------------------------------------
 static constexpr int CMS_MAX = 32;           // atoms
@@ -632,7 +632,7 @@ __global__ __launch_bounds__(CM_WAVE) void atomic_cm_kernel(
 // is by rank, as in cm_small_kernel, where that is the repeated selection's: no NaN key, and no
 // picked key equal to the value that marks picked atoms.
 // Bound by instruction issue, then by writing the rows: 140,000 rows of size 23 in distance order
-// 713 -> 129 us = 2.4 TB/s, row-norm order 1145 -> 162.
+// 699 -> 126 us = 2.6 TB/s, row-norm order 1145 -> 162.
 static constexpr int ACMS_MAX_CHUNK = 16;
 static_assert(QMLH_ACM_SMALL_ATOMS == CMS_MAX, "one lane per atom");
 

@@ -29,9 +29,11 @@ static constexpr int GK_TILE = WG_T;
 
 // Kernel matrices of fewer than this many 128 x 128 tiles are computed in 64 x 64 ones (four times
 // the workgroups): with few tiles the launch lasts as long as one tile, and later the last round
-// leaves less of the chip idle. Symmetric Gaussian, 435 features, n = 1000 / 4500 / 8000 / 10007:
-// 87 / 279 / 570 / 988 us on 128 x 128 tiles, 29 / 229 / 558 / 948 on 64 x 64; at 6241 tiles (the
-// linear kernel of 10007 x 10007) 1561 against 1580.
+// leaves less of the chip idle, which fades as the rounds grow. 435 features, 128 x 128 against 64 x
+// 64 tiles, us: symmetric Gaussian, 36 tiles 87 / 29, 666 279 / 229, 2556 709 / 679, 3741 1047 / 996,
+// 5253 1456 / 1401, 7021 1915 / 1873; Gaussian of two sets, 1024 tiles 274 / 266, 3969 1072 / 1007,
+// 8836 2323 / 2259; linear, 3025 732 / 730, 6557 1570 / 1570. The line is not sharp: beyond it the
+// Gaussian would still gain 2 to 5 % and the linear kernel of two sets nothing.
 static constexpr int64_t GK_SMALL_TILES = 4096;
 
 static int64_t kernel_tiles(int64_t na, int64_t nb, bool sym, int64_t side) {

@@ -435,8 +435,7 @@ __device__ __forceinline__ void wg_tile_mma_lds(WaveTile<T, Q>& t, T* __restrict
 // C(row0 + 16 b + (lane & 15), col0 + tile_row(a, e)) (first operand = output columns).
 // `live`: the wave's block has entries to update; `interior`: every entry of its block
 // is inside the M x N matrix (and on or below the diagonal when LOWER), so no masks are needed
-// and all loads are issued back to back. Masked entries load as zero and are not stored; nor are
-// rows below first_row (an interior block has none).
+// and all loads are issued back to back. Masked entries load as zero and are not stored.
 // ------------------------------------------------------------------------------------------
 template <typename T, bool LOWER, int Q>
 __device__ __forceinline__ void wave_tile_load_c(WaveTile<T, Q>& t, const T* __restrict__ C,
@@ -469,8 +468,7 @@ __device__ __forceinline__ void wave_tile_load_c(WaveTile<T, Q>& t, const T* __r
 template <typename T, bool LOWER, int Q>
 __device__ __forceinline__ void wave_tile_store_c(const WaveTile<T, Q>& t, T* __restrict__ C,
                                                   int64_t ldc, int64_t row0, int64_t col0,
-                                                  int64_t M, int64_t N, bool interior,
-                                                  int64_t first_row = 0) {
+                                                  int64_t M, int64_t N, bool interior) {
     const int lane = threadIdx.x & 63;
     if (interior) {
 #pragma unroll
@@ -487,7 +485,7 @@ __device__ __forceinline__ void wave_tile_store_c(const WaveTile<T, Q>& t, T* __
 #pragma unroll
         for (int b = 0; b < Q; ++b) {
             const int64_t i = row0 + 16 * b + (lane & 15);
-            if (i >= M || i < first_row) continue;
+            if (i >= M) continue;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int64_t j = col0 + tile_row<T>(a, e);

@@ -68,12 +68,6 @@ __global__ __launch_bounds__(PT_THREADS, 2) void pair_tile_kernel(
     }
 }
 
-// Tile rows: with few 128 x 128 tiles a launch lasts as long as one tile, so 64- and 32-row tiles
-// spread it over more CUs, at more operand reads per pair. Laplacian kernel, 276 features, 128- /
-// 64- / 32-row tiles: 64 tiles (1000 x 1000) 101 / 60 / 42 us, 121 tiles 105 / 64 / 61, 225 tiles
-// 110 / 99 / 110, 576 tiles 240 / 211 / 221, 1024 tiles 339 / 350 / 388.
-static constexpr int64_t PAIR_TILES_64 = 800, PAIR_TILES_32 = 160;
-
 template <int OP, int EPI, int R>
 static void launch_pair_tiles(const double* A, int64_t na, int64_t lda, const double* B, int64_t nb,
                               int64_t ldb, int64_t d, const PairEpi& ep, double* K, int64_t ldk,

@@ -89,6 +89,13 @@ __device__ __forceinline__ double pair_epilogue(double acc, const PairEpi& e) {
     return acc;
 }
 
+// Tile rows: with few 128 x 128 tiles a launch lasts as long as one tile, so 64- and 32-row tiles
+// spread it over more CUs, at more operand reads per pair. Laplacian kernel, 276 features, 128- /
+// 64- / 32-row tiles: 64 tiles (1000 x 1000) 101 / 60 / 42 us, 121 tiles 105 / 64 / 61, 225 tiles
+// 110 / 99 / 110, 576 tiles 240 / 211 / 221, 1024 tiles 339 / 350 / 388. Launches of fewer 128 x 128
+// tiles than these take 64- and 32-row ones.
+static constexpr int64_t PAIR_TILES_64 = 800, PAIR_TILES_32 = 160;
+
 // LDS of a tile: two buffers of a k-major chunk of each operand.
 static constexpr int PT_ELEMS = 2 * 2 * PT_BK * PT_LDS;
 

@@ -300,10 +300,10 @@ static int predict_impl(int32_t kind, const double* Xq, int64_t m, int64_t ldq,
                                s, Xq, ldq, m, normsQ, Xt, ldt, n, normsT, alpha, d, scale, part);
     } else {
         // Query rows per tile: no more than the queries need, and small tiles where few of the
-        // large ones would leave CUs idle (the pairwise kernels' line; whole call with 4 queries,
+        // large ones would leave CUs idle (the pairwise kernels' lines; whole call with 4 queries,
         // 2,952 rows: 209 us on 128-row tiles, 132 on 32).
         const int64_t tiles = ceil_div(m, 128) * nchunks;
-        const int R = m <= 32 || tiles < 160 ? 2 : m <= 64 || tiles < 800 ? 4 : 8;
+        const int R = m <= 32 || tiles < PAIR_TILES_32 ? 2 : m <= 64 || tiles < PAIR_TILES_64 ? 4 : 8;
         auto kernel = R == 2 ? predict_laplace_kernel<2>
                              : R == 4 ? predict_laplace_kernel<4> : predict_laplace_kernel<8>;
         hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(m, 16 * R), (unsigned)nchunks),
