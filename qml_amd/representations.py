@@ -114,7 +114,9 @@ def generate_atomic_coulomb_matrices_device(Zd, Rd, Od, central, cmol, size: int
     rows = central.shape[0]
     if out is None:
         out = torch.empty((rows, ld), dtype=torch.float64, device=Od.device)
-    status = torch.zeros(1, dtype=torch.int32, device=Od.device)
+    # the second word is the 32-lane kernel's own status; it lives as long as the caller's
+    words = torch.zeros(2, dtype=torch.int32, device=Od.device)
+    status = words[:1]
     L = _lib.lib()
     args = (_lib.ptr(Zd), _lib.ptr(Rd), _lib.ptr(Od), Od.shape[0] - 1, _lib.ptr(central),
             _lib.ptr(cmol), rows, size, _ACM_SORTINGS[sorting], float(central_cutoff),
@@ -125,7 +127,7 @@ def generate_atomic_coulomb_matrices_device(Zd, Rd, Od, central, cmol, size: int
         max_atoms = int((Od[1:] - Od[:-1]).max()) if Od.shape[0] > 1 else 0
     if max_atoms <= _lib.ACM_SMALL_ATOMS:
         small = max(0, int(max_atoms))
-        first = torch.zeros(1, dtype=torch.int32, device=Od.device) if hinted else status
+        first = words[1:] if hinted else status
         _lib.check(L.qmlh_atomic_cm_small(*args, _lib.ptr(first), small,
                                           _lib.stream_handle(stream)))
         if hinted:  # a molecule may still be larger than the caller says

@@ -51,3 +51,15 @@ def test_status_of_both_kernels():
                                                        max_atoms=m) for m in (10, 256)]
         assert [int(s) for _, s in got] == [want, want]
         assert bool((got[0][0] == got[1][0]).all())
+
+
+def test_status_keeps_the_first_kernels_word():
+    """On a stream of the caller's own the second launch reads it after the call has returned."""
+    import torch
+
+    from qml_amd.representations import generate_atomic_coulomb_matrices_device
+
+    batch = _batch([12, 40])
+    status = generate_atomic_coulomb_matrices_device(*batch, 40, max_atoms=10)[1]
+    assert status.shape == (1,) and status.dtype == torch.int32
+    assert status.untyped_storage().nbytes() == 8
