@@ -198,8 +198,7 @@ __device__ __forceinline__ void lk_panel_atoms(LkPanel& P, int nm, int a0, int t
 typedef PanelLoader<double, LAYOUT_ROW, 4, true> LkRows;
 template <bool WIDE>
 __device__ __forceinline__ LkRows lk_rows(const LkPanel& P, const LkSide& S) {
-    return LkRows(S.X, S.ld, P.row, S.order ? P.lowest : P.row[0],
-                  S.order ? (int)S.atoms - 1 : P.row[LK_TILE - 1], WIDE);
+    return LkRows(S.X, S.ld, P.row, S.order ? P.lowest : P.row[0], WIDE);
 }
 
 // Add this wave's molecule-pair sums of one sigma to S.

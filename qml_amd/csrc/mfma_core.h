@@ -221,10 +221,11 @@ struct PanelLoader {
             last_row = false;
         }
     }
-    // The rows of X listed in rows[0 .. 32 Q - 1] (LDS), from `first` to `highest` (the same in every
-    // lane). wide: they span 4 GiB or more.
+    // The rows of X listed in rows[0 .. 32 Q - 1] (LDS), none below `first` (the same in every lane).
+    // wide: they span 4 GiB or more. The caller holds them to X: the view's length does not (it
+    // would be one more scalar register in kernels that spill them).
     __device__ __forceinline__ PanelLoader(const T* X, int64_t ldx, const int* rows, int first,
-                                           int highest, bool wide) {
+                                           bool wide) {
         static_assert(LISTED && LAYOUT == LAYOUT_ROW, "rows are listed for row-major operands");
         const int lane = threadIdx.x & 63;
         const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -235,7 +236,7 @@ struct PanelLoader {
         by_value = wide;
         base = X + uniform_i64(first * ldx);
         step = 1;
-        bytes = (uint32_t)uniform_i64(((highest - first) * ldx + WG_KC) * (int64_t)sizeof(T));
+        bytes = 0xffffffffu;
 #pragma unroll
         for (int u = 0; u < Q; ++u) {
             const int row = 8 * Q * wave + 8 * u + (lane >> 3);
