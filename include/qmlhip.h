@@ -504,6 +504,12 @@ int qmlh_local_kernels_ordered(int32_t kind, const double *A, int64_t atomsA, in
                                int64_t ldk, int64_t sstride, int32_t flags, void *ws,
                                size_t ws_bytes, qmlh_stream_t stream);
 
+/* counts (device, npA int32) := per panel 1 + the last feature that is not zero in any of its
+ * atoms' rows: what an order of the molecules would let qmlh_local_kernels_ordered skip. */
+int qmlh_local_feature_counts(const double *A, int64_t atomsA, int64_t lda, const int64_t *offsA,
+                              const int64_t *panelsA, const int64_t *orderA, int64_t npA,
+                              int64_t d, int32_t *counts, qmlh_stream_t stream);
+
 /* Panel partition for qmlh_local_kernels (host only, no device work; no counterpart in the
  * reference, whose loops run molecule pair by molecule pair): consecutive molecules are grouped
  * into panels of at most QMLH_LOCAL_PANEL_ATOMS atoms and QMLH_LOCAL_PANEL_MOLS molecules; a

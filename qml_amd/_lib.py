@@ -73,6 +73,8 @@ _SIGNATURES = {
     "qmlh_local_kernels_ordered": (ctypes.c_int, [
         _i32, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _i64,
         _i64, _vp, _i32, _vp, _i64, _i64, _i32, _vp, _sz, _vp]),
+    "qmlh_local_feature_counts": (ctypes.c_int, [_vp, _i64, _i64, _vp, _vp, _vp, _i64, _i64, _vp,
+                                                 _vp]),
     "qmlh_local_panels": (_i64, [_vp, _i64, _vp]),
     "qmlh_pairwise": (ctypes.c_int, [_i32, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _f64, _vp,
                                      _i64, _i32, _vp]),

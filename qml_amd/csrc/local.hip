@@ -15,7 +15,8 @@
 // size 23 (276 features), the mean over
 // panel pairs is 199 features for differences and 105 for products, against 264 and 230 in random
 // order. 4,000 such molecules, Gaussian by differences, three widths: 42.9 -> 33.5 ms; 3,000 x 701,
-// Laplacian: 9.98 -> 7.50 ms. A workgroup computes the atom-pair distance tile of its panel
+// Laplacian: 9.98 -> 7.50 ms. (Without padding to skip, an order only makes more panels and scatters
+// their rows, 5 to 40 % of a call: the caller weighs that, from qmlh_local_feature_counts.) A workgroup computes the atom-pair distance tile of its panel
 // pair (128 x 128 atoms: FP64 MFMA expanded form for the Gaussian, the FP64 VALU direct tile
 // for the Laplacian and the direct Gaussian), applies exp for each sigma, and reduces the tile
 // to molecule-pair sums with two small MFMA products against 0/1 membership matrices:
@@ -77,33 +78,38 @@ __device__ __forceinline__ int lk_features(const LkSide& A, const LkSide& B, int
     return f < d ? f : (int)d;
 }
 
-// count[panel] := 1 + the last feature that is not zero in any of the panel's atom rows, with
-// LK_NOT_FINITE where FINITE asks for it. One workgroup per panel, four wavefronts per molecule and
-// four molecules at a time: a wavefront's rows are one memory latency after the other.
-template <bool FINITE>
-__global__ __launch_bounds__(LK_COUNT_LANES) void local_feature_counts_kernel(LkSide A, int64_t npanels,
-                                                                   int64_t d,
-                                                                   int32_t* __restrict__ count) {
+// count[panel] := 1 + the last feature that is not zero in any of the panel's atom rows, for the
+// panels of side A and then of side B. With norms (products), LK_NOT_FINITE is set where one of the
+// panel's is not finite, as it is when a value is not (and when finite ones overflow it: then all
+// features are taken without need). One workgroup per panel, four wavefronts per molecule and four
+// molecules at a time: a wavefront's rows are one memory latency after the other. Rows are read from
+// the end up to their last nonzero feature; a kernel per side that read all of them to see whether
+// they are finite took 20,000 molecules of 276 features from 618 (Laplacian) to 631 ms and from
+// 253 (Gaussian) to 255.
+__global__ __launch_bounds__(LK_COUNT_LANES) void local_feature_counts_kernel(
+    LkSide A, int64_t npA, LkSide B, int64_t npB, int64_t d, int32_t* __restrict__ count) {
     constexpr int WAVES = LK_COUNT_LANES / 64;
     __shared__ int s_last[WAVES], s_bad[WAVES];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int64_t panel = blockIdx.x; panel < npanels; panel += gridDim.x) {
+    for (int64_t p = blockIdx.x; p < npA + npB; p += gridDim.x) {
+        const LkSide& S = p < npA ? A : B;
+        const int64_t panel = p < npA ? p : p - npA;
         int last = 0, bad = 0;  // per wave
-        for (int64_t m = A.panels[panel] + wave / 4; m < A.panels[panel + 1]; m += WAVES / 4) {
-            const int64_t mol = A.order ? A.order[m] : m;
-            for (int64_t r = A.offsets[mol] + wave % 4; r < A.offsets[mol + 1]; r += 4) {
-                const double* x = A.X + r * A.ld;
-                // from the end, 64 features at a time; without FINITE no further than `last`
-                for (int64_t k0 = (d - 1) / 64 * 64; k0 >= 0 && (FINITE || k0 + 64 > last); k0 -= 64) {
+        for (int64_t m = S.panels[panel] + wave / 4; m < S.panels[panel + 1]; m += WAVES / 4) {
+            const int64_t mol = S.order ? S.order[m] : m;
+            for (int64_t r = S.offsets[mol] + wave % 4; r < S.offsets[mol + 1]; r += 4) {
+                const double* x = S.X + r * S.ld;
+                if (S.norms) bad |= !(fabs(S.norms[r]) <= DBL_MAX);
+                // from the end, 64 features at a time, no further than `last`
+                for (int64_t k0 = (d - 1) / 64 * 64; k0 >= 0 && k0 + 64 > last; k0 -= 64) {
                     const int64_t k = k0 + lane;
                     const double v = k < d ? x[k] : 0.0;
                     const unsigned long long nz = __ballot(v != 0.0);
                     if (nz) {
                         const int top = (int)k0 + 64 - __builtin_clzll(nz);
                         last = top > last ? top : last;
+                        break;
                     }
-                    if (FINITE) bad |= __any(!(fabs(v) <= DBL_MAX));
-                    if (!FINITE && nz) break;
                 }
             }
         }
@@ -118,7 +124,7 @@ __global__ __launch_bounds__(LK_COUNT_LANES) void local_feature_counts_kernel(Lk
                 l = s_last[w] > l ? s_last[w] : l;
                 b |= s_bad[w];
             }
-            count[panel] = l | (FINITE && b ? LK_NOT_FINITE : 0);
+            count[p] = l | (b ? LK_NOT_FINITE : 0);
         }
         __syncthreads();
     }
@@ -435,6 +441,13 @@ extern "C" int64_t qmlh_local_panels(const int64_t* offsets_h, int64_t nmol, int
 
 namespace qmlh {
 
+static void launch_counts(const LkSide& A, int64_t npA, const LkSide& B, int64_t npB, int64_t d,
+                          int32_t* counts, hipStream_t s) {
+    const int64_t panels = npA + npB, most = 16384;
+    hipLaunchKernelGGL(local_feature_counts_kernel, dim3((unsigned)(panels < most ? panels : most)),
+                       dim3(LK_COUNT_LANES), 0, s, A, npA, B, npB, d, counts);
+}
+
 // counts: (npA + npB) int32 for the panels' feature counts, or null to use all features.
 static int local_kernels(int32_t kind, const double* A, int64_t atomsA, int64_t lda,
                          const double* normsA, const int64_t* offsA, const int64_t* panelsA,
@@ -482,16 +495,10 @@ static int local_kernels(int32_t kind, const double* A, int64_t atomsA, int64_t 
     // the counts and 119 without; 400 x 20, two widths, 164 and 130. 3,000 x 701: 6.97 ms with
     // counts by 16 wavefronts a panel, 7.11 by four.
     if (counts && (symmetric ? npA * (npA + 1) / 2 : npA * npB) > LK_COUNT_PAIRS) {
+        launch_counts(sa, npA, sb, symmetric ? 0 : npB, d, counts, s);
+        QMLH_CHECK_LAUNCH("local_kernels feature counts launch");
         sa.count = counts;
         sb.count = symmetric ? counts : counts + npA;
-        auto launch = mfma ? local_feature_counts_kernel<true> : local_feature_counts_kernel<false>;
-        const int64_t most = 16384;
-        hipLaunchKernelGGL(launch, dim3((unsigned)(npA < most ? npA : most)), dim3(LK_COUNT_LANES), 0, s, sa,
-                           npA, d, counts);
-        if (!symmetric)
-            hipLaunchKernelGGL(launch, dim3((unsigned)(npB < most ? npB : most)), dim3(LK_COUNT_LANES), 0, s,
-                               sb, npB, d, counts + npA);
-        QMLH_CHECK_LAUNCH("local_kernels feature counts launch");
     }
     for (int32_t s0 = 0; s0 < nsig; s0 += LK_NS) {
         LkSigmas sg;
@@ -526,6 +533,22 @@ extern "C" int qmlh_local_kernels(int32_t kind, const double* A, int64_t atomsA,
     return qmlh::local_kernels(kind, A, atomsA, lda, normsA, offsA, panelsA, nullptr, npA, B,
                                atomsB, ldb, normsB, offsB, panelsB, nullptr, npB, d, sigmas_h,
                                nsig, K, ldk, sstride, flags, nullptr, stream);
+}
+
+extern "C" int qmlh_local_feature_counts(const double* A, int64_t atomsA, int64_t lda,
+                                         const int64_t* offsA, const int64_t* panelsA,
+                                         const int64_t* orderA, int64_t npA, int64_t d,
+                                         int32_t* counts, qmlh_stream_t stream) {
+    using namespace qmlh;
+    if (npA < 0 || atomsA < 0 || d < 0 || lda < d)
+        return set_error(QMLH_ERR_ARG, "local_feature_counts: bad shape");
+    if (npA == 0) return QMLH_OK;
+    if ((atomsA > 0 && !A) || !offsA || !panelsA || !counts)
+        return set_error(QMLH_ERR_ARG, "local_feature_counts: null pointer");
+    const LkSide side{A, lda, nullptr, offsA, panelsA, orderA, nullptr, atomsA};
+    launch_counts(side, npA, side, 0, d, counts, (hipStream_t)stream);
+    QMLH_CHECK_LAUNCH("local_feature_counts launch");
+    return QMLH_OK;
 }
 
 extern "C" size_t qmlh_local_kernels_workspace(int64_t npA, int64_t npB) {

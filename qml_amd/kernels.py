@@ -236,6 +236,10 @@ def local_panels(offsets) -> np.ndarray:
     return panels[:np_ + 1].copy()
 
 
+# Features from which a set's order by size is weighed against its own order (_local_orders).
+ORDER_FEATURES = 128
+
+
 class LocalSet:
     """Atom representations of a molecule list resident in HBM, with what the local-kernel
     launch needs: rows (atoms, ld) FP64, atom offsets on the device, the molecules ordered by
@@ -271,8 +275,28 @@ class LocalSet:
         self.offsets_d, self.panels_d, self.own_panels_d, order_d = (
             buf[e - p.size:e] for p, e in zip(parts, ends))
         self.order_d = order_d if order.size else None
+        self.skipping = self._skipping()
         self._norms = None
         self._maxnorm = None
+
+    def _skipping(self):
+        """What the order by size gives a call of more than LOCAL_COUNT_PAIRS panel pairs, from the
+        rows as they are now: (panels per panel of the own order, mean over panel pairs of the
+        features that a product needs, and that a difference needs); None where no such call takes
+        it. It needs the rows' lengths on the host, some 40 us once a set."""
+        import torch
+
+        n, own = self.panels.size - 1, self.own_panels.size - 1
+        if self.order_d is None or self.d < ORDER_FEATURES or n * n <= _lib.LOCAL_COUNT_PAIRS:
+            return None
+        counts = torch.empty(n, dtype=torch.int32, device=self.X.device)
+        _lib.check(_lib.lib().qmlh_local_feature_counts(
+            _lib.ptr(self.X), self.atoms, self.X.shape[1], _lib.ptr(self.offsets_d),
+            _lib.ptr(self.panels_d), _lib.ptr(self.order_d), n, self.d, _lib.ptr(counts),
+            _lib.stream_handle()))
+        c = np.sort(counts.cpu().numpy()).astype(np.float64)
+        rank = 2.0 * np.arange(n) + 1.0  # pairs (of n^2) whose larger count is c[i]
+        return n / own, float(c @ rank[::-1]) / n ** 2, float(c @ rank) / n ** 2
 
     @property
     def npanels(self) -> int:
@@ -290,19 +314,37 @@ class LocalSet:
         return self._maxnorm
 
 
-def _local_orders(SA: LocalSet, SB: LocalSet, symmetric: bool):
-    """(order, panels) of both sides for a call. Up to LOCAL_COUNT_PAIRS panel pairs no padding is
-    skipped, and an order by size only makes more panels (16 small molecules do not fill one), so
-    such a call takes the molecules' own order where that has no more panel pairs: 192 molecules of
-    5 to 23 atoms are 253 pairs and not 276, one round of the 256 CUs and not two."""
+# A panel pair's time beyond its features, in features, by products and by differences (from 60 and
+# 276 features without zeros: 59 and 167 ns a pair, 84 and 302).
+PAIR_FEATURES = {True: 58.0, False: 23.0}
+
+
+def _local_orders(SA: LocalSet, SB: LocalSet, symmetric: bool, product: bool):
+    """(order, panels) of both sides for a call, in the molecules' own order or by size. By size the
+    panels are more (16 small molecules do not fill one), their rows scattered and the features
+    counted: a call takes it where that has fewer panel pairs, or where enough trailing zeros are
+    skipped, which no call of up to LOCAL_COUNT_PAIRS panel pairs does. 5 to 23 atoms, 276 features,
+    175 molecules are 253 pairs in their own order and not 276, one round of the 256 CUs and not two.
+    Products and differences in us, in the own order and by size: 875 such molecules with padding
+    895 and 1598, 546 and 1338; without 944 and 1684, 973 and 1661 (130 features, 1312 molecules of 8
+    to 15 atoms: 620 and 1020, 466 and 862; 629 and 1020, 720 and 1091). Rows shorter than
+    ORDER_FEATURES skip too little: 60 features, 1909 molecules of 5 to 10 atoms, 505 and 712, 477
+    and 689; without padding 507 and 714, 632 and 838."""
     def pairs(a, b):
         return a * (a + 1) // 2 if symmetric else a * b
 
-    ordered = pairs(SA.panels.size - 1, SB.panels.size - 1)
-    if ordered <= _lib.LOCAL_COUNT_PAIRS and \
-            pairs(SA.own_panels.size - 1, SB.own_panels.size - 1) <= ordered:
-        return [(None, S.own_panels_d) for S in (SA, SB)]
-    return [(S.order_d, S.panels_d) for S in (SA, SB)]
+    sizes = pairs(SA.panels.size - 1, SB.panels.size - 1)
+    own = pairs(SA.own_panels.size - 1, SB.own_panels.size - 1)
+    known = [S.skipping for S in (SA, SB) if S.skipping is not None]
+    by_size = sizes < own
+    if sizes > _lib.LOCAL_COUNT_PAIRS and known:  # a set of few panels is taken for the other's like
+        more = known[0][0] * known[-1][0]
+        need = np.sqrt(known[0][1 if product else 2] * known[-1][1 if product else 2])
+        fixed = PAIR_FEATURES[product]
+        by_size = more * (fixed + need) < 0.9 * (fixed + SA.d)
+    if by_size:
+        return [(S.order_d, S.panels_d) for S in (SA, SB)]
+    return [(None, S.own_panels_d) for S in (SA, SB)]
 
 
 def local_kernels_device(kind: int, SA: LocalSet, SB: LocalSet, sigmas, symmetric=False,
@@ -329,8 +371,16 @@ def local_kernels_device(kind: int, SA: LocalSet, SB: LocalSet, sigmas, symmetri
         if expanded:
             nA, nB = SA.norms(), SB.norms()
     L = _lib.lib()
-    (oA, pA), (oB, pB) = _local_orders(SA, SB, symmetric)
+    (oA, pA), (oB, pB) = _local_orders(SA, SB, symmetric, nA is not None)
     npA, npB = pA.numel() - 1, pB.numel() - 1
+    if oA is None and oB is None:
+        _lib.check(L.qmlh_local_kernels(
+            kind, _lib.ptr(SA.X), SA.atoms, SA.X.shape[1], _lib.ptr(nA), _lib.ptr(SA.offsets_d),
+            _lib.ptr(pA), npA, _lib.ptr(SB.X), SB.atoms, SB.X.shape[1], _lib.ptr(nB),
+            _lib.ptr(SB.offsets_d), _lib.ptr(pB), npB, SA.d, sig.ctypes.data, sig.size,
+            _lib.ptr(K), SA.nmol, SA.nmol * SB.nmol, _lib.SYMMETRIC if symmetric else 0,
+            _lib.stream_handle(stream)))
+        return K
     ws_bytes = L.qmlh_local_kernels_workspace(npA, npB)
     with torch.cuda.stream(stream) if stream is not None else contextlib.nullcontext():
         ws = torch.empty(max(1, (ws_bytes + 7) // 8), dtype=torch.float64, device=SA.X.device)

@@ -10,12 +10,13 @@ LINE = 512  # panel pairs up to which the features are not counted
 
 
 def _rows(counts, d, ld, seed):
-    """Rows of each molecule: nonzero up to a length that grows with its size, then zeros."""
+    """Rows of each molecule: nonzero up to a length that grows with its size (all features from 23
+    atoms), then zeros."""
     rng = np.random.default_rng(seed)
     X = np.zeros((int(np.sum(counts)), ld))
     r = 0
     for n in counts:
-        length = min(d, 1 + 3 * int(n))
+        length = d if n >= 23 else min(d, 1 + 3 * int(n))
         X[r:r + n, :length] = rng.random((n, length)) * 5
         r += n
     return X
@@ -46,10 +47,11 @@ FORMS = [("gaussian", True), ("gaussian", False), ("laplacian", False)]
 
 def _check(kind, expanded, A, B, symmetric):
     from qml_amd import _lib
-    from qml_amd.kernels import local_kernels_device
+    from qml_amd.kernels import _local_orders, local_kernels_device
 
     pairs = A.npanels * (A.npanels + 1) // 2 if symmetric else A.npanels * B.npanels
     assert pairs > LINE
+    assert _local_orders(A, B, symmetric, expanded)[0][0] is not None  # and so the features counted
     k = _lib.PAIR_GAUSSIAN if kind == "gaussian" else _lib.PAIR_LAPLACIAN
     sig = np.array([6.0, 20.0])
     got = local_kernels_device(k, A, B, sig, symmetric, expanded=expanded)
@@ -63,7 +65,7 @@ def _check(kind, expanded, A, B, symmetric):
 
 @pytest.mark.parametrize("kind,expanded", FORMS)
 @pytest.mark.parametrize("symmetric", [True, False])
-@pytest.mark.parametrize("d,ld", [(70, 80), (64, 64), (65, 80)])
+@pytest.mark.parametrize("d,ld", [(139, 144), (128, 128), (129, 144)])
 def test_skipped_features(kind, expanded, symmetric, d, ld):
     import torch
 
@@ -89,7 +91,7 @@ def test_values_that_are_not_finite(kind, expanded, symmetric, value):
 
     from qml_amd.kernels import LocalSet
 
-    d, ld, mol = 70, 80, 17
+    d, ld, mol = 139, 144, 17
     na = np.random.default_rng(3).integers(1, 24, size=600)
     na[mol] = 23
     X = _rows(na, d, ld, 1)
