@@ -993,7 +993,8 @@ static int atomic_cm_rows(const char* who, const double* Z, const double* R,
     if (nrows == 0) return QMLH_OK;
     if (!Z || !R || !offsets || !central || !cmol || !out)
         return set_error(QMLH_ERR_ARG, "%s: null pointer", who);
-    TimerScope ts(QMLH_TIMER_CM, (double)nrows, s);
+    // the rows were counted by the first kernel's launch
+    TimerScope ts(first ? -1 : QMLH_TIMER_CM, (double)nrows, s);
     hipLaunchKernelGGL((sorting == QMLH_ACM_ROW_NORM ? atomic_cm_kernel<true>
                                                      : atomic_cm_kernel<false>),
                        dim3((unsigned)(nrows < grid ? nrows : grid)), dim3(CM_WAVE), 0, s, Z, R,

@@ -63,3 +63,18 @@ def test_status_keeps_the_first_kernels_word():
     status = generate_atomic_coulomb_matrices_device(*batch, 40, max_atoms=10)[1]
     assert status.shape == (1,) and status.dtype == torch.int32
     assert status.untyped_storage().nbytes() == 8
+
+
+def test_rows_are_timed_once():
+    """The launch that looks for rows left over counts none of its own: a call with a hint is one
+    launch of its rows to the timers, as a call without."""
+    from qml_amd import _lib
+    from qml_amd.representations import generate_atomic_coulomb_matrices_device
+
+    batch = _batch([5, 12, 23])
+    for hint in (None, 23):
+        _lib.timer_enable(True)
+        generate_atomic_coulomb_matrices_device(*batch, 23, max_atoms=hint)
+        _, launches, rows = _lib.timer_read("cm")
+        _lib.timer_enable(False)
+        assert (launches, rows) == (1, 40)
